@@ -71,6 +71,8 @@ def lib():
             "gpeed_dtype_block_size": ([i32], i32),
             "gpeed_dtype_row_bytes": ([i32, u64], sz),
             "gpeed_matmul_rows": ([i32, vp, u64, u64, i32, i32, vp, i32, vp, vp], i32),
+            "gpeed_matmul_rows_ws_bytes": ([i32, i64, i64, i32], sz),
+            "gpeed_matmul_rows_ws": ([i32, vp, u64, u64, i32, i32, vp, i32, vp, vp, sz, vp], i32),
             "gpeed_codebook": ([i32, vp, sz], i32),
             "gpeed_t64_grid_table": ([vp, sz], i32),
             "gpeed_t64_aux_word": ([C.c_uint32], C.c_uint32),
@@ -682,8 +684,19 @@ def matmul_rows(dtype: int, w, n_rows: int, row0: int, in_dim: int, out_dim: int
     n_tok = X2.shape[0]
     if out is None:
         out = torch.empty((n_tok, out_dim), dtype=torch.float32, device=X.device)
-    _check(lib().gpeed_matmul_rows(dtype, _ptr(w), n_rows, row0, in_dim, out_dim, _ptr(X2), n_tok, _ptr(out),
-                                   _stream(stream)), "matmul_rows")
+    need = lib().gpeed_matmul_rows_ws_bytes(dtype, in_dim, out_dim, n_tok)
+    if need:
+        # X in operand order: scratch of this call, of the stream that it runs on
+        if stream is None:
+            ws = torch.empty(need, dtype=torch.uint8, device=X.device)
+        else:
+            with torch.cuda.stream(stream):
+                ws = torch.empty(need, dtype=torch.uint8, device=X.device)
+        _check(lib().gpeed_matmul_rows_ws(dtype, _ptr(w), n_rows, row0, in_dim, out_dim, _ptr(X2), n_tok, _ptr(out),
+                                          _ptr(ws), need, _stream(stream)), "matmul_rows")
+    else:
+        _check(lib().gpeed_matmul_rows(dtype, _ptr(w), n_rows, row0, in_dim, out_dim, _ptr(X2), n_tok, _ptr(out),
+                                       _stream(stream)), "matmul_rows")
     return out.reshape(out_dim) if vec else out
 
 

@@ -356,9 +356,8 @@ int gpeed_dequantize(int dtype, const void* src, float* dst, uint64_t n, gpeed_s
     return e == hipSuccess ? GPEED_OK : hip_fail(e, "dequantize launch");
 }
 
-int gpeed_matmul_rows(int dtype, const void* w, uint64_t n_rows, uint64_t row0, int in_dim, int out_dim,
-                      const float* X, int n_tok, float* Y, gpeed_stream_t stream) {
-    if (n_tok <= 0 || out_dim <= 0) return GPEED_OK;  // weights.cpp:88
+static int check_rows_args(int dtype, const void* w, uint64_t n_rows, uint64_t row0, int in_dim, int out_dim,
+                           const float* X, int n_tok, float* Y) {
     const int be = gpeed::rows_block_elems(dtype);
     if (be == 0) return fail(GPEED_ERR_UNIMPLEMENTED, "matmul_rows: unimplemented type " + std::to_string(dtype));
     // the block formats' kernels walk rows in 32-weight runs; F32 rows (in
@@ -371,14 +370,49 @@ int gpeed_matmul_rows(int dtype, const void* w, uint64_t n_rows, uint64_t row0, 
         return fail(GPEED_ERR_INVALID, "matmul_rows: rows [row0, row0 + out_dim) outside the tensor");
     if (!aligned(w, dtype == GPEED_DTYPE_F32 ? 4 : 2) || !aligned(X, 16) || !aligned(Y, 4))
         return fail(GPEED_ERR_INVALID, "matmul_rows: w element-aligned, X 16-byte and Y 4-byte aligned");
-    const size_t rb = gpeed_dtype_row_bytes(dtype, (uint64_t)in_dim);
-    hipError_t e = gpeed::launch_matmul_rows(dtype, static_cast<const uint8_t*>(w), rb, row0, in_dim, out_dim, X,
-                                             n_tok, Y, static_cast<hipStream_t>(stream));
+    return GPEED_OK;
+}
+
+static int rows_status(hipError_t e) {
     // (the type is known here, so the only invalid value left is a row
     // length whose per-wavefront row group passes the 2 GiB offset range)
     if (e == hipErrorInvalidValue)
         return fail(GPEED_ERR_INVALID, "matmul_rows: rows too long (one wavefront's rows exceed 2 GiB)");
     return e == hipSuccess ? GPEED_OK : hip_fail(e, "matmul_rows launch");
+}
+
+int gpeed_matmul_rows(int dtype, const void* w, uint64_t n_rows, uint64_t row0, int in_dim, int out_dim,
+                      const float* X, int n_tok, float* Y, gpeed_stream_t stream) {
+    if (n_tok <= 0 || out_dim <= 0) return GPEED_OK;  // weights.cpp:88
+    const int rc = check_rows_args(dtype, w, n_rows, row0, in_dim, out_dim, X, n_tok, Y);
+    if (rc) return rc;
+    return rows_status(gpeed::launch_matmul_rows(dtype, static_cast<const uint8_t*>(w),
+                                                 gpeed_dtype_row_bytes(dtype, (uint64_t)in_dim), row0, in_dim, out_dim,
+                                                 X, n_tok, Y, static_cast<hipStream_t>(stream)));
+}
+
+size_t gpeed_matmul_rows_ws_bytes(int dtype, int64_t in_dim, int64_t out_dim, int n_tok) {
+    const int be = gpeed::rows_block_elems(dtype);
+    if (be == 0 || in_dim <= 0 || in_dim > (1 << 28) || in_dim % be || in_dim % 32 || out_dim <= 0 ||
+        out_dim > INT_MAX || n_tok <= 0 || n_tok > (1 << 24))
+        return 0;
+    return gpeed::rows_gemm_ws_bytes(dtype, (int)in_dim, (int)out_dim, n_tok);
+}
+
+int gpeed_matmul_rows_ws(int dtype, const void* w, uint64_t n_rows, uint64_t row0, int in_dim, int out_dim,
+                         const float* X, int n_tok, float* Y, void* ws, size_t ws_bytes, gpeed_stream_t stream) {
+    if (n_tok <= 0 || out_dim <= 0) return GPEED_OK;
+    const int rc = check_rows_args(dtype, w, n_rows, row0, in_dim, out_dim, X, n_tok, Y);
+    if (rc) return rc;
+    const size_t need = gpeed_matmul_rows_ws_bytes(dtype, in_dim, out_dim, n_tok);
+    if (need && (!ws || ws_bytes < need || !aligned(ws, 256)))
+        return fail(GPEED_ERR_INVALID, "matmul_rows: workspace null, too small or not 256-byte aligned");
+    const uint8_t* wp = static_cast<const uint8_t*>(w);
+    const size_t rb = gpeed_dtype_row_bytes(dtype, (uint64_t)in_dim);
+    const hipStream_t s = static_cast<hipStream_t>(stream);
+    return rows_status(need ? gpeed::launch_rows_gemm(dtype, wp, rb, row0, in_dim, out_dim, X, n_tok, Y,
+                                                      static_cast<uint8_t*>(ws), s)
+                            : gpeed::launch_matmul_rows(dtype, wp, rb, row0, in_dim, out_dim, X, n_tok, Y, s));
 }
 
 int gpeed_codebook(int dtype, uint64_t* out, size_t n) {

@@ -30,6 +30,13 @@ size_t rows_block_bytes(int dtype);
 hipError_t launch_dequant_rows(int dtype, const uint8_t* src, float* dst, unsigned long long n, hipStream_t s);
 hipError_t launch_matmul_rows(int dtype, const uint8_t* w, size_t row_bytes, unsigned long long row0, int in_dim,
                               int out_dim, const float* X, int n_tok, float* Y, hipStream_t s);
+// The same products for many tokens on the fp16 matrix cores
+// (quant_gemm.hip), with a workspace for X in operand order:
+// rows_gemm_ws_bytes bytes, 16-byte aligned, no initialisation (0: this type
+// and token count run without one, through launch_matmul_rows).
+size_t rows_gemm_ws_bytes(int dtype, int in_dim, int out_dim, int n_tok);
+hipError_t launch_rows_gemm(int dtype, const uint8_t* w, size_t row_bytes, unsigned long long row0, int in_dim,
+                            int out_dim, const float* X, int n_tok, float* Y, uint8_t* ws, hipStream_t s);
 uint64_t rows_iq2s_grid(int i);
 uint32_t rows_iq3s_grid(int i);
 // Streaming read of `bytes` from p (16-byte aligned) by n_groups workgroups;

@@ -14,270 +14,11 @@
 // workgroup.
 #include "iq3_common.h"
 #include "iq3_kernels.h"
-#include "quant_grids.h"
-
-#include <type_traits>
+#include "quant_decode.h"
 
 namespace gpeed {
 
 namespace {
-
-constexpr int kDtF32 = 0, kDtF16 = 1, kDtQ8_0 = 8, kDtQ2_K = 10, kDtQ3_K = 11, kDtQ6_K = 14, kDtIQ3_XXS = 18,
-              kDtIQ3_S = 21, kDtIQ2_S = 22, kDtIQ4_XS = 23, kDtBF16 = 30;
-
-struct Iq2sGrid { uint64_t v[1024]; };
-struct Iq3sGrid { uint32_t v[512]; };
-constexpr uint16_t kIq2sPacked[1024] = {GPEED_IQ2S_PACKED};
-constexpr uint16_t kIq3sPacked[512] = {GPEED_IQ3S_PACKED};
-constexpr uint8_t kIq2sLevel[3] = {GPEED_IQ2S_LEVELS};
-constexpr int8_t kIq4nl[16] = {GPEED_IQ4NL_VALUES};
-
-constexpr Iq2sGrid expand_iq2s() {
-    Iq2sGrid g{};
-    for (int i = 0; i < 1024; ++i) {
-        uint64_t e = 0;
-        for (int j = 0; j < 8; ++j) e |= (uint64_t)kIq2sLevel[(kIq2sPacked[i] >> (2 * j)) & 3] << (8 * j);
-        g.v[i] = e;
-    }
-    return g;
-}
-constexpr Iq3sGrid expand_iq3s() {
-    Iq3sGrid g{};
-    for (int i = 0; i < 512; ++i) {
-        uint32_t e = 0;
-        for (int j = 0; j < 4; ++j) e |= (2u * ((kIq3sPacked[i] >> (3 * j)) & 7u) + 1u) << (8 * j);
-        g.v[i] = e;
-    }
-    return g;
-}
-constexpr Iq2sGrid kIq2sGrid = expand_iq2s();
-constexpr Iq3sGrid kIq3sGrid = expand_iq3s();
-
-// Geometry (quant.cpp:52-114): weights per block, bytes per block. Scalar
-// types are handled in 32-weight runs.
-template <int DT> struct Fmt;
-template <> struct Fmt<kDtF32> { static constexpr int kElems = 32, kBytes = 128; };
-template <> struct Fmt<kDtF16> { static constexpr int kElems = 32, kBytes = 64; };
-template <> struct Fmt<kDtBF16> { static constexpr int kElems = 32, kBytes = 64; };
-template <> struct Fmt<kDtQ8_0> { static constexpr int kElems = 32, kBytes = 34; };
-template <> struct Fmt<kDtQ2_K> { static constexpr int kElems = 256, kBytes = 84; };
-template <> struct Fmt<kDtQ3_K> { static constexpr int kElems = 256, kBytes = 110; };
-template <> struct Fmt<kDtQ6_K> { static constexpr int kElems = 256, kBytes = 210; };
-template <> struct Fmt<kDtIQ3_XXS> { static constexpr int kElems = 256, kBytes = 98; };
-template <> struct Fmt<kDtIQ3_S> { static constexpr int kElems = 256, kBytes = 110; };
-template <> struct Fmt<kDtIQ2_S> { static constexpr int kElems = 256, kBytes = 82; };
-template <> struct Fmt<kDtIQ4_XS> { static constexpr int kElems = 256, kBytes = 136; };
-
-// Codebook copies in LDS (only the one the format uses is sized).
-template <int DT>
-struct Tables {
-    static constexpr int kN = DT == kDtIQ2_S ? 1024 : DT == kDtIQ3_S ? 512 : DT == kDtIQ3_XXS ? 256 : 16;
-    using T = typename std::conditional<DT == kDtIQ2_S, uint64_t, uint32_t>::type;
-    T v[kN];
-    __device__ void load(int tid, int nthreads) {
-        for (int i = tid; i < kN; i += nthreads) {
-            if constexpr (DT == kDtIQ2_S) v[i] = kIq2sGrid.v[i];
-            else if constexpr (DT == kDtIQ3_S) v[i] = kIq3sGrid.v[i];
-            else if constexpr (DT == kDtIQ3_XXS) v[i] = kIq3xxsGrid[i];
-            else v[i] = (uint32_t)(int32_t)kIq4nl[i];
-        }
-    }
-};
-
-// Loads of block fields: blocks sit at 2-byte-aligned addresses (every
-// block size is even), so wider fields are assembled from 16-bit loads.
-__device__ __forceinline__ uint32_t u8(const uint8_t* p) { return *p; }
-__device__ __forceinline__ uint32_t u16(const uint8_t* p) { return *reinterpret_cast<const uint16_t*>(p); }
-__device__ __forceinline__ uint32_t u32a2(const uint8_t* p) { return u16(p) | (u16(p + 2) << 16); }
-// 32 bytes from a 2-byte-aligned address as 8 little-endian words
-__device__ __forceinline__ void bytes32(const uint8_t* p, uint32_t (&w)[8]) {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) w[i] = u32a2(p + 4 * i);
-}
-__device__ __forceinline__ uint32_t byte_of(const uint32_t (&w)[8], int i) { return (w[i >> 2] >> (8 * (i & 3))) & 255u; }
-
-// decode32: weights 32*sb .. 32*sb+31 of the block at blk into y. Each
-// formula restates the reference's block function for those weights; the
-// comment gives its lines and the byte layout.
-template <int DT>
-__device__ __forceinline__ void decode32(const uint8_t* __restrict__ blk, int sb, const Tables<DT>& tb, float (&y)[32]) {
-#pragma clang fp contract(off)
-    if constexpr (DT == kDtF32) {
-        // quant.cpp:528-531: a copy
-        const float* f = reinterpret_cast<const float*>(blk);
-#pragma unroll
-        for (int i = 0; i < 32; ++i) y[i] = f[i];
-    } else if constexpr (DT == kDtF16 || DT == kDtBF16) {
-        // quant.cpp:532-545 (f16_to_f32 :130-154, bf16_to_f32 :156-161); the
-        // hardware fp16 conversion is exact (subnormals included)
-#pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            const uint32_t h = u16(blk + 2 * i);
-            y[i] = DT == kDtF16 ? (float)__builtin_bit_cast(_Float16, (uint16_t)h) : __uint_as_float(h << 16);
-        }
-    } else if constexpr (DT == kDtQ8_0) {
-        // quant.cpp:165-184: d (fp16), 32 int8 codes; y = d * q
-        const float d = f16_bits_to_f32(u16(blk));
-        uint32_t w[8];
-        bytes32(blk + 2, w);
-#pragma unroll
-        for (int i = 0; i < 32; ++i) y[i] = d * (float)(int8_t)byte_of(w, i);
-    } else if constexpr (DT == kDtQ6_K) {
-        // quant.cpp:212-306: ql[128] qh[64] sc[16] d. Sub-block sb: half
-        // h = sb/4, quarter q = sb%4; weight l < 32 takes the low (q < 2)
-        // or high nibble of ql[64h + 32(q&1) + l], bits 2q of qh[32h + l],
-        // scale sc[8h + 2q + l/16]; y = (d * sc) * (v - 32).
-        const int h = sb >> 2, q = sb & 3;
-        const float d = f16_bits_to_f32(u16(blk + 208));
-        const float ds0 = d * (float)(int8_t)u8(blk + 192 + 8 * h + 2 * q);
-        const float ds1 = d * (float)(int8_t)u8(blk + 192 + 8 * h + 2 * q + 1);
-        uint32_t lo[8], hi[8];
-        bytes32(blk + 64 * h + 32 * (q & 1), lo);
-        bytes32(blk + 128 + 32 * h, hi);
-#pragma unroll
-        for (int l = 0; l < 32; ++l) {
-            const uint32_t b = byte_of(lo, l);
-            const uint32_t nib = q >= 2 ? b >> 4 : b & 15u;
-            const int v = (int)(nib | (((byte_of(hi, l) >> (2 * q)) & 3u) << 4)) - 32;
-            y[l] = (l < 16 ? ds0 : ds1) * (float)v;
-        }
-    } else if constexpr (DT == kDtQ2_K) {
-        // quant.cpp:309-335: scales[16] qs[64] d dmin. Sub-block sb: half
-        // h = sb/4, plane j = sb%4; weight l < 32: code (qs[32h + l] >> 2j)
-        // & 3, scale byte scales[8h + 2j + l/16];
-        // y = (d * (sc & 15)) * code - dmin * (sc >> 4).
-        const int h = sb >> 2, j = sb & 3;
-        const float d = f16_bits_to_f32(u16(blk + 80));
-        const float mn = f16_bits_to_f32(u16(blk + 82));
-        const uint32_t s0 = u8(blk + 8 * h + 2 * j), s1 = u8(blk + 8 * h + 2 * j + 1);
-        const float dl0 = d * (float)(s0 & 15u), ml0 = mn * (float)(s0 >> 4);
-        const float dl1 = d * (float)(s1 & 15u), ml1 = mn * (float)(s1 >> 4);
-        uint32_t w[8];
-        bytes32(blk + 16 + 32 * h, w);
-#pragma unroll
-        for (int l = 0; l < 32; ++l) {
-            const float c = (float)((byte_of(w, l) >> (2 * j)) & 3u);
-            y[l] = l < 16 ? dl0 * c - ml0 : dl1 * c - ml1;
-        }
-    } else if constexpr (DT == kDtQ3_K) {
-        // quant.cpp:337-370: hmask[32] qs[64] scales[12] d. Sub-block sb:
-        // h = sb/4, j = sb%4; weight l < 32: code (qs[32h + l] >> 2j) & 3,
-        // minus 4 where bit 4h + j of hmask[l] is clear; 6-bit scale k =
-        // 8h + 2j + l/16 unpacked from the 12 bytes (low nibble of byte k,
-        // or high nibble of byte k-8 for k >= 8; top bits from byte 8 + k%4
-        // at 2*(k/4)); y = (d * (scale - 32)) * value.
-        const int h = sb >> 2, j = sb & 3;
-        const float d = f16_bits_to_f32(u16(blk + 108));
-        float dl[2];
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const int k = 8 * h + 2 * j + s;
-            const uint32_t low = k < 8 ? u8(blk + 96 + k) & 15u : u8(blk + 96 + k - 8) >> 4;
-            const uint32_t top = (u8(blk + 104 + (k & 3)) >> (2 * (k >> 2))) & 3u;
-            dl[s] = d * (float)((int)(int8_t)(uint8_t)(low | (top << 4)) - 32);
-        }
-        uint32_t w[8], m[8];
-        bytes32(blk + 32 + 32 * h, w);
-        bytes32(blk, m);
-#pragma unroll
-        for (int l = 0; l < 32; ++l) {
-            const int code = (int)((byte_of(w, l) >> (2 * j)) & 3u);
-            const int v = code - (((byte_of(m, l) >> (4 * h + j)) & 1u) ? 0 : 4);
-            y[l] = dl[l >> 4] * (float)v;
-        }
-    } else if constexpr (DT == kDtIQ3_XXS) {
-        // quant.cpp:186-210: d, qs[64] grid indices, 8 words of 4 x 7 sign
-        // bits + 4-bit scale; the eighth sign of a group makes the parity
-        // even. y = ((d * (0.5 + s)) * 0.5) * grid * sign.
-        const float d = f16_bits_to_f32(u16(blk));
-        const uint32_t aux = u32a2(blk + 66 + 4 * sb);
-        const float db = d * (0.5f + (float)(aux >> 28)) * 0.5f;
-#pragma unroll
-        for (int l = 0; l < 4; ++l) {
-            const uint32_t qq = u16(blk + 2 + 8 * sb + 2 * l);
-            const uint32_t s7 = (aux >> (7 * l)) & 127u;
-            const uint32_t sg = s7 | ((__builtin_popcount(s7) & 1u) << 7);
-            const uint32_t g1 = tb.v[qq & 255u], g2 = tb.v[qq >> 8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t gv = ((e < 4 ? g1 : g2) >> (8 * (e & 3))) & 255u;
-                y[8 * l + e] = db * (float)gv * (((sg >> e) & 1u) ? -1.0f : 1.0f);
-            }
-        }
-    } else if constexpr (DT == kDtIQ2_S) {
-        // quant.cpp:373-418: d, qs[32] grid low bytes, signs[32], qh[8],
-        // scales[8]. Group l < 4 of sub-block sb: index qs[4sb + l] | bits
-        // 2l, 2l+1 of qh[sb] as bits 8-9; scale nibble (low for l < 2) of
-        // scales[sb]; y = ((d * (0.5 + s)) * 0.25) * grid * sign, sign bit e
-        // of signs[4sb + l].
-        const float d = f16_bits_to_f32(u16(blk));
-        const uint32_t qh = u8(blk + 66 + sb), sc = u8(blk + 74 + sb);
-        const float db0 = d * (0.5f + (float)(sc & 15u)) * 0.25f;
-        const float db1 = d * (0.5f + (float)(sc >> 4)) * 0.25f;
-        const uint32_t qs = u32a2(blk + 2 + 4 * sb), sg = u32a2(blk + 34 + 4 * sb);
-#pragma unroll
-        for (int l = 0; l < 4; ++l) {
-            const uint32_t idx = ((qs >> (8 * l)) & 255u) | ((qh << (8 - 2 * l)) & 0x300u);
-            const uint64_t g = tb.v[idx];
-            const uint32_t s = sg >> (8 * l);
-            const float dl = l < 2 ? db0 : db1;
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                y[8 * l + e] = dl * (float)(uint32_t)((g >> (8 * e)) & 255u) * (((s >> e) & 1u) ? -1.0f : 1.0f);
-        }
-    } else if constexpr (DT == kDtIQ3_S) {
-        // quant.cpp:421-482: d, qs[64], qh[8], signs[32], scales[4]. Group
-        // l < 4 of sub-block sb: indices qs[8sb + 2l], qs[8sb + 2l + 1] with
-        // bit 8 from bits 2l and 2l+1 of qh[sb]; scale nibble of
-        // scales[sb/2] (low for even sb); y = (d * (1 + 2s)) * grid * sign,
-        // sign bit e of signs[4sb + l].
-        const float d = f16_bits_to_f32(u16(blk));
-        const uint32_t qh = u8(blk + 66 + sb);
-        const uint32_t scb = u8(blk + 106 + (sb >> 1));
-        const float db = d * (1.0f + 2.0f * (float)((sb & 1) ? scb >> 4 : scb & 15u));
-        const uint32_t sg = u32a2(blk + 74 + 4 * sb);
-#pragma unroll
-        for (int l = 0; l < 4; ++l) {
-            const uint32_t qq = u16(blk + 2 + 8 * sb + 2 * l);
-            const uint32_t i1 = (qq & 255u) | ((qh << (8 - 2 * l)) & 256u);
-            const uint32_t i2 = (qq >> 8) | ((qh << (7 - 2 * l)) & 256u);
-            const uint32_t g1 = tb.v[i1], g2 = tb.v[i2];
-            const uint32_t s = sg >> (8 * l);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t gv = ((e < 4 ? g1 : g2) >> (8 * (e & 3))) & 255u;
-                y[8 * l + e] = db * (float)gv * (((s >> e) & 1u) ? -1.0f : 1.0f);
-            }
-        }
-    } else if constexpr (DT == kDtIQ4_XS) {
-        // quant.cpp:485-502: d, scales_h (u16), scales_l[4], qs[128].
-        // Sub-block sb: 6-bit scale = nibble sb%2 of scales_l[sb/2] | bits
-        // 2sb, 2sb+1 of scales_h << 4; weight i < 16 is the low nibble of
-        // qs[16sb + i], weight 16 + i its high nibble;
-        // y = (d * (ls - 32)) * level[code].
-        const float d = f16_bits_to_f32(u16(blk));
-        const uint32_t sh = u16(blk + 2);
-        const int ls = (int)(((u8(blk + 4 + (sb >> 1)) >> (4 * (sb & 1))) & 15u) | (((sh >> (2 * sb)) & 3u) << 4));
-        const float dl = d * (float)(ls - 32);
-        uint32_t w[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = u32a2(blk + 8 + 16 * sb + 4 * i);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const uint32_t b = (w[i >> 2] >> (8 * (i & 3))) & 255u;
-            y[i] = dl * (float)(int32_t)tb.v[b & 15u];
-            y[16 + i] = dl * (float)(int32_t)tb.v[b >> 4];
-        }
-    }
-}
-
-// Sub-blocks per block and the sub-block's block address.
-template <int DT>
-__device__ __forceinline__ const uint8_t* sub_block(const uint8_t* row, long long sbi, int& sb) {
-    constexpr int kSub = Fmt<DT>::kElems / 32;
-    sb = (int)(sbi % kSub);
-    return row + (size_t)(sbi / kSub) * Fmt<DT>::kBytes;
-}
 
 // One thread per 32-weight sub-block, grid-stride; y written as 8 float4.
 template <int DT>

@@ -123,7 +123,7 @@ void WeightStore::read_resident(const std::string& name, void* dst) const {
 WeightStore::~WeightStore() {
     for (auto& kv : tensors_) (void)gpeed_free(kv.second.data);
     for (auto& kv : ws_) (void)gpeed_free(kv.second.p);
-    for (Buffer* b : {&x_, &y_, &route_ws_, &moe_ws_, &batch_ws_, &logits_, &bias_, &eptr_, &tok_, &wt_})
+    for (Buffer* b : {&x_, &y_, &rows_ws_, &route_ws_, &moe_ws_, &batch_ws_, &logits_, &bias_, &eptr_, &tok_, &wt_})
         (void)gpeed_free(b->p);
 }
 
@@ -273,9 +273,11 @@ void WeightStore::rows_product(const Tensor& t, const std::string& name, uint64_
     const size_t xb = (size_t)n_tok * in_dim * sizeof(float), yb = (size_t)n_tok * out_dim * sizeof(float);
     void* xd = scratch(x_, xb, false);
     void* yd = scratch(y_, yb, false);
+    const size_t wsb = gpeed_matmul_rows_ws_bytes(t.dtype, in_dim, out_dim, n_tok);
+    void* ws = wsb ? scratch(rows_ws_, wsb, false) : nullptr;
     check(gpeed_memcpy(xd, X, xb, kH2D), "weights: upload x");
-    check(gpeed_matmul_rows(t.dtype, t.data, t.n_rows, row0, in_dim, out_dim, static_cast<const float*>(xd), n_tok,
-                            static_cast<float*>(yd), nullptr),
+    check(gpeed_matmul_rows_ws(t.dtype, t.data, t.n_rows, row0, in_dim, out_dim, static_cast<const float*>(xd), n_tok,
+                               static_cast<float*>(yd), ws, wsb, nullptr),
           ("weights: product over " + name).c_str());
     check(gpeed_memcpy(Y, yd, yb, kD2H), "weights: download y");
 }

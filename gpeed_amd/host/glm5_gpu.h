@@ -173,7 +173,7 @@ private:
     // it is made and grown when a call needs more; each launch leaves its
     // tickets at zero, and one sized for n_tok serves every smaller call.
     std::map<std::tuple<int, int>, Buffer> ws_;
-    Buffer x_, y_, route_ws_, moe_ws_, batch_ws_, logits_, bias_, eptr_, tok_, wt_, mlp_ws_;
+    Buffer x_, y_, rows_ws_, route_ws_, moe_ws_, batch_ws_, logits_, bias_, eptr_, tok_, wt_, mlp_ws_;
 };
 
 }  // namespace gpu

@@ -164,6 +164,16 @@ size_t gpeed_dtype_row_bytes(int dtype, uint64_t n);
  * every type. */
 int gpeed_matmul_rows(int dtype, const void* w, uint64_t n_rows, uint64_t row0, int in_dim, int out_dim,
                       const float* X, int n_tok, float* Y, gpeed_stream_t stream);
+/* The same product with a workspace: from a few tokens on (F32 rows excepted)
+ * X is laid out once in the workspace and the product runs on the fp16 matrix
+ * cores with weights and activations as fp16 hi and lo parts, its error
+ * against exact arithmetic no larger than gpeed_matmul_rows'. ws: device
+ * memory of gpeed_matmul_rows_ws_bytes bytes, 256-byte aligned, no
+ * initialisation, one per stream; the size 0 means that this type and token
+ * count need none (ws may be NULL; the call is gpeed_matmul_rows'). */
+size_t gpeed_matmul_rows_ws_bytes(int dtype, int64_t in_dim, int64_t out_dim, int n_tok);
+int gpeed_matmul_rows_ws(int dtype, const void* w, uint64_t n_rows, uint64_t row0, int in_dim, int out_dim,
+                         const float* X, int n_tok, float* Y, void* ws, size_t ws_bytes, gpeed_stream_t stream);
 /* Host-only (no reference counterpart): the expanded codebook the kernels
  * use for IQ2_S (1024 entries of 8 bytes), IQ3_S (512 of 4) or IQ3_XXS
  * (256 of 4), one entry per uint64. */
