@@ -345,7 +345,9 @@ hipError_t matmul_dt_nt(const uint8_t* w, size_t rb, int in_dim, int out_dim, co
         const uint8_t* wj = w + (size_t)j * rb;
         const uint8_t* base = reinterpret_cast<const uint8_t*>(reinterpret_cast<uintptr_t>(wj) & ~(uintptr_t)15);
         const uint32_t lead = (uint32_t)(wj - base);
-        const int base_bytes = (int)(lead + (size_t)rows * rb);
+        // to the end of the last bytes' dword: a dword past the range in part
+        // reads as zero
+        const int base_bytes = (int)((lead + (size_t)rows * rb + 3) & ~(size_t)3);
         int grid = (rows + 4 * RW - 1) / (4 * RW);
         if (grid > 2048) grid = 2048;
         for (int t = 0; t < n_tok; t += kMaxTok) {

@@ -111,6 +111,18 @@ def test_non_finite_values(gpu, dt, rows, n_tok):
         1e-30).expand_as(ref)[ok]).max()) < TIGHT
 
 
+@pytest.mark.parametrize("dt", [8, 11, 18, 21, 22])
+@pytest.mark.parametrize("n_tok", [1, 3])
+def test_last_row_ends_inside_a_dword(gpu, dt, n_tok):
+    """Few-token slices over an odd number of rows of 2 bytes more than whole
+    dwords: the last row's last bytes count."""
+    in_dim, rows = (160, 127) if dt == 8 else (256, 127)
+    w = synth.quant_matrix(65, dt, dt, rows, in_dim)
+    X = synth.normal(65, n_tok, n_tok * in_dim).reshape(n_tok, in_dim)
+    Y = G.matmul_rows(dt, dev(w.reshape(-1), gpu), rows, 0, in_dim, rows, dev(X, gpu)).cpu().numpy()
+    assert rel_err(Y, oracle.matmul_rows(dt, w, 0, in_dim, rows, X)) < TIGHT
+
+
 def test_captured_and_on_another_stream(gpu):
     """A captured call replays (no launch depends on host state), and a call on
     a stream of its own matches."""
