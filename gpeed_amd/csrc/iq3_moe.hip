@@ -11,9 +11,9 @@
 //                SwiGLU of the gate/up rows) into its segment's prepared
 //                activation.
 // k_gemv_grouped ragged grouped GEMV: a wavefront takes (segment, tensor,
-//                tile) items (its first by its index, the others from an
-//                atomic counter) and streams the tile's records over the
-//                whole row (no partial sums leave it).
+//                tile) items, one a round, and streams the tile's records
+//                over the whole row, or (few tokens) over a part of it, whose
+//                sums the next launch adds.
 // k_moe_combine  Y[t] = sum over the token's slots, in expert order, of
 //                wt * down row (one fma per term, like axpy_f32).
 #include <algorithm>
@@ -349,7 +349,7 @@ struct MoePlan {
     int* slot_tok;   // [N + T_sh] token of slot p (gather-mode activations)
     int* pos;        // [T][K] slots of token t, in expert order
     int* pos_tmp;    // [T][K] the same, unordered (global scratch of the stand-alone plan)
-    uint32_t* ctr;   // [3] work counters (gate/up, down) and the whole-step front kernel's ticket
+    uint32_t* ctr;   // the whole-step front kernel's ticket (word 2)
     uint32_t* err;   // the workspace's error word (kWsBuckets)
 };
 
@@ -429,9 +429,6 @@ __device__ __forceinline__ void plan_body(const int* eptr, const int* tok, int T
             base += ccount[c];
         }
         *pl.n_seg = base;
-        // the grouped GEMVs take work from these with device-scope atomics
-        __hip_atomic_store(pl.ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(pl.ctr + 1, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
     for (int e = tid; e < E && segs; e += 1024) {
@@ -535,14 +532,23 @@ __device__ __forceinline__ BlockImages block_images(const float (&e)[4]) {
     return r;
 }
 
+__device__ __forceinline__ void add4(float4& a, const float4& b) {
+    a.x += b.x;
+    a.y += b.y;
+    a.z += b.z;
+    a.w += b.w;
+}
+
 // One wavefront per (slot p, block b). MODE 0: v = X[tok[p]]; MODE 1:
 // v = silu(min(G[p],lim)) * clamp(U[p],-lim,lim), over the bucket slots and
-// then the n_extra shared-expert slots.
+// then the n_extra shared-expert slots; G and U in `parts` planes of
+// part_stride floats, added in order.
 template <int MODE>
 __global__ __launch_bounds__(256) void k_prep_grouped(const float* __restrict__ X, const float* __restrict__ U,
                                                       const int* __restrict__ tok, const int* __restrict__ eptr,
                                                       int E, int nb, float lim, MoePlan pl,
-                                                      uint8_t* __restrict__ act, size_t seg_stride, int n_extra) {
+                                                      uint8_t* __restrict__ act, size_t seg_stride, int n_extra,
+                                                      int parts, size_t part_stride) {
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int item = blockIdx.x * 4 + wave;
     const int N = *pl.n_valid + (*pl.n_seg > 0 ? n_extra : 0);
@@ -550,10 +556,14 @@ __global__ __launch_bounds__(256) void k_prep_grouped(const float* __restrict__ 
     const int p = item / nb, b = item - p * nb;
     const size_t row = MODE == 0 ? (size_t)tok[p] : (size_t)p;
     const size_t src = row * nb * 256 + (size_t)b * 256 + 4 * lane;
-    const float4 v = *reinterpret_cast<const float4*>(X + src);
+    float4 v = *reinterpret_cast<const float4*>(X + src);
+    if (MODE == 1) {
+        for (int q = 1; q < parts; ++q) add4(v, *reinterpret_cast<const float4*>(X + q * part_stride + src));
+    }
     float e[4] = {v.x, v.y, v.z, v.w};
     if (MODE == 1) {
-        const float4 u = *reinterpret_cast<const float4*>(U + src);
+        float4 u = *reinterpret_cast<const float4*>(U + src);
+        for (int q = 1; q < parts; ++q) add4(u, *reinterpret_cast<const float4*>(U + q * part_stride + src));
         const float us[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -682,9 +692,10 @@ struct GroupedArgs {
     int nb;                   // blocks per row
     int tiles;                // 64-row tiles per expert
     int tiles_per_item;       // consecutive row tiles one work item streams (divides tiles)
+    int parts;                // or (tiles_per_item 1) the items a row tile's blocks are cut into
+    size_t part_stride;       // floats between the sums of consecutive parts in y
     int rows;                 // rows per expert (= output width)
     MoePlan pl;
-    int ctr_index;
     int n_exp;                // expert id of the shared expert's segments
     // gather mode: activations are per-token images (token_images), read
     // through the slots' tokens, instead of per-segment images
@@ -722,17 +733,19 @@ __device__ __forceinline__ void load_record_gather(Rec<NP>& r, const uint8_t* re
 // nt consecutive row tiles (records rec0 .. rec0 + nt*nb - 1, tile-major) of
 // one segment: the ring runs on across the tile boundaries; each tile's sums
 // go to y at its end.
+// An item that is a part of one tile (nt 1) walks the tile's nbt blocks from
+// b0 on (rec0: its first record); else nbt = nb and b0 = 0.
 // kGather: the activations come from per-token images (timg, tus) through
 // slot_tok[p0 ..], not from the segment's own images at act.
 template <int NP, bool kGather>
 __device__ __forceinline__ void grouped_tile(const uint8_t* tbl, uint32_t lb, uint32_t lane, const uint8_t* rec0,
-                                             const uint8_t* act, int n, int nb, int nt, float* y, int rows,
-                                             int row0, const uint8_t* timg, const float* tus,
+                                             const uint8_t* act, int n, int nb, int b0, int nbt, int nt, float* y,
+                                             int rows, int row0, const uint8_t* timg, const float* tus,
                                              const int* slot_tok, int p0) {
     // records in flight: two, or one for four token pairs (a record and its
     // activation images take 58 registers there; two of them spilled)
     constexpr int PF = NP >= 4 ? 1 : 2;
-    const int nrec = nt * nb;
+    const int nrec = nt * nbt;
     const float* xsc = reinterpret_cast<const float*>(act + (size_t)nb * n * 1024);
     // The block unscales travel with the record ring: one wait per record
     // covers both, where a load issued at the product would expose its
@@ -752,7 +765,7 @@ __device__ __forceinline__ void grouped_tile(const uint8_t* tbl, uint32_t lb, ui
     }
     auto fill = [&](Rec<NP>& r, int k) {  // record k of the item (clamped to the last)
         k = min(k, nrec - 1);
-        const int b = k % nb;
+        const int b = b0 + k % nbt;
         if constexpr (kGather) {
             load_record_gather<NP>(r, rec0 + (size_t)k * kRecordBytes, timg + (size_t)b * 1024, toff, lane);
             r.xs = __builtin_bit_cast(uint32_t, tus[us_row + b]);
@@ -787,7 +800,7 @@ __device__ __forceinline__ void grouped_tile(const uint8_t* tbl, uint32_t lb, ui
 #pragma unroll
                 for (int t = 0; t < 2 * NP; ++t)
                     if (t < n) acc[t] = fmaf(d4 * rec_unscale(ring[s], t), blk[t], acc[t] + dz);
-                if (++kb == nb) {  // uniform
+                if (++kb == nbt) {  // uniform
 #pragma unroll
                     for (int t = 0; t < 2 * NP; ++t) {
                         if (t < n) y[(size_t)t * rows + row0 + tile * kTileRows + lane] = acc[t];
@@ -815,30 +828,38 @@ __global__ __launch_bounds__(kGroupedThreads, 2) void k_gemv_grouped(GroupedArgs
     grid_table_store<kGroupedThreads>(tbl, gw, tid);
     lds_barrier();
     const int groups = g.tiles / g.tiles_per_item;  // items per segment and tensor
-    const int per_seg = g.n_tensors * groups;
+    const int per_seg = g.n_tensors * groups * g.parts;
     const int n_items = *g.pl.n_seg * per_seg;
-    // the first round is static (wavefront i takes item i), the rest come
-    // from the counter: 2048 wavefronts taking tickets on one address at
-    // once serialise for tens of microseconds
+    // Static rounds in snake order: wavefront i takes item i, then the i-th
+    // from the end of the second round, and so on. Segments are numbered
+    // heaviest first, so a wavefront's items even out. A counter on one address
+    // hands items out no better and makes every wavefront wait for its last,
+    // empty ticket (steps of 1 / 8 / 32 tokens, 64 experts top-8, hidden 6144,
+    // inter 2048: 88 / 180 / 309 us with tickets, 74 / 166 / 288 without).
     constexpr int kWavesPerGroup = kGroupedThreads / 64;
     const uint32_t n_waves = gridDim.x * kWavesPerGroup;
-    uint32_t item = blockIdx.x * kWavesPerGroup + (tid >> 6);
+    const uint32_t wave0 = blockIdx.x * kWavesPerGroup + (tid >> 6);
+    uint32_t item = wave0, round = 0;
     while (true) {
         if (item >= (uint32_t)n_items) break;
         const int s = item / per_seg;
-        const int rem = item - s * per_seg;
+        int rem = item - s * per_seg;
+        const int part = rem % g.parts;
+        rem /= g.parts;
+        const int b0 = g.nb * part / g.parts, nbt = g.nb * (part + 1) / g.parts - b0;
         const int ten = rem / groups, tile = (rem - ten * groups) * g.tiles_per_item;
         const int e = g.pl.seg_e[s], p0 = g.pl.seg_p0[s], n = g.pl.seg_n[s];
-        const uint8_t* rec0 = e == g.n_exp ? g.w_sh[ten] + (size_t)tile * g.nb * kRecordBytes
-                                           : g.w[ten] + ((size_t)e * g.tiles + tile) * g.nb * kRecordBytes;
+        const uint8_t* rec0 = (e == g.n_exp ? g.w_sh[ten] + (size_t)tile * g.nb * kRecordBytes
+                                            : g.w[ten] + ((size_t)e * g.tiles + tile) * g.nb * kRecordBytes) +
+                              (size_t)b0 * kRecordBytes;
         const uint8_t* act = g.act + (size_t)s * g.seg_stride;
-        float* y = g.y[ten] + (size_t)p0 * g.rows;
+        float* y = g.y[ten] + part * g.part_stride + (size_t)p0 * g.rows;
         const int nt = g.tiles_per_item;
-#define GPEED_GROUPED_TILE(NP)                                                                                   \
-    (g.timg ? grouped_tile<NP, true>(tbl, lb, lane, rec0, act, n, g.nb, nt, y, g.rows, tile * kTileRows, g.timg, \
-                                     g.tus, g.pl.slot_tok, p0)                                                   \
-            : grouped_tile<NP, false>(tbl, lb, lane, rec0, act, n, g.nb, nt, y, g.rows, tile * kTileRows,       \
-                                      nullptr, nullptr, nullptr, 0))
+#define GPEED_GROUPED_TILE(NP)                                                                        \
+    (g.timg ? grouped_tile<NP, true>(tbl, lb, lane, rec0, act, n, g.nb, b0, nbt, nt, y, g.rows,       \
+                                     tile * kTileRows, g.timg, g.tus, g.pl.slot_tok, p0)              \
+            : grouped_tile<NP, false>(tbl, lb, lane, rec0, act, n, g.nb, b0, nbt, nt, y, g.rows,      \
+                                      tile * kTileRows, nullptr, nullptr, nullptr, 0))
         switch ((n + 1) >> 1) {
             case 1: GPEED_GROUPED_TILE(1); break;
             case 2: GPEED_GROUPED_TILE(2); break;
@@ -846,9 +867,8 @@ __global__ __launch_bounds__(kGroupedThreads, 2) void k_gemv_grouped(GroupedArgs
             default: GPEED_GROUPED_TILE(4); break;
         }
 #undef GPEED_GROUPED_TILE
-        uint32_t t = 0;
-        if (lane == 0) t = __hip_atomic_fetch_add(g.pl.ctr + g.ctr_index, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        item = n_waves + __builtin_amdgcn_readfirstlane(__shfl(t, 0));
+        ++round;
+        item = round * n_waves + ((round & 1) ? n_waves - 1 - wave0 : wave0);
     }
 }
 
@@ -857,11 +877,12 @@ __global__ __launch_bounds__(kGroupedThreads, 2) void k_gemv_grouped(GroupedArgs
 // slots in expert order, one fma per term.
 // With the shared expert (sh: its down rows, one per token; model_batch.cpp:
 // 264-280), Y[t] = that sum + sh[t] (add_f32), unless the plan rejected
-// the buckets (n_seg 0).
+// the buckets (n_seg 0). D (and sh) in `parts` planes of part_stride floats,
+// added in order.
 __global__ __launch_bounds__(256) void k_moe_combine(const float* __restrict__ D, const float* __restrict__ wt,
                                                      const int* __restrict__ pos, int T, int K, int H,
                                                      float* __restrict__ Y, const float* __restrict__ sh,
-                                                     const int* __restrict__ n_seg) {
+                                                     const int* __restrict__ n_seg, int parts, size_t part_stride) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     const size_t n4 = (size_t)T * H / 4;
     if (i >= n4) return;
@@ -872,14 +893,17 @@ __global__ __launch_bounds__(256) void k_moe_combine(const float* __restrict__ D
         const int p = pos[(size_t)t * K + k];
         if (p < 0) continue;  // buckets rejected by the plan
         const float w = wt[p];
-        const float4 d = *reinterpret_cast<const float4*>(D + (size_t)p * H + h);
+        float4 d = *reinterpret_cast<const float4*>(D + (size_t)p * H + h);
+        for (int q = 1; q < parts; ++q) add4(d, *reinterpret_cast<const float4*>(D + q * part_stride + (size_t)p * H + h));
         y.x = fmaf(w, d.x, y.x);
         y.y = fmaf(w, d.y, y.y);
         y.z = fmaf(w, d.z, y.z);
         y.w = fmaf(w, d.w, y.w);
     }
     if (sh && *n_seg > 0) {
-        const float4 d = *reinterpret_cast<const float4*>(sh + (size_t)t * H + h);
+        float4 d = *reinterpret_cast<const float4*>(sh + (size_t)t * H + h);
+        for (int q = 1; q < parts; ++q)
+            add4(d, *reinterpret_cast<const float4*>(sh + q * part_stride + (size_t)t * H + h));
         y.x = y.x + d.x;
         y.y = y.y + d.y;
         y.z = y.z + d.z;
@@ -906,6 +930,38 @@ struct MoeLayout {
 // from 9 tokens one GEMM pass beats two GEMV passes.
 constexpr int kMoeGemmMinAvg = 9;
 bool moe_use_gemm(int T, int E, int K) { return (long long)T * K >= (long long)kMoeGemmMinAvg * E; }
+
+// Slot rows the gate, up and down sums take: room for up to
+// kMaxParts parts of few slots (never less for more slots, so a workspace
+// serves every smaller call).
+constexpr int kMaxParts = 4;
+constexpr size_t kPartRows = 640;
+size_t part_rows(size_t slots) { return std::max(slots, std::min(kMaxParts * slots, kPartRows)); }
+
+// How a grouped GEMV over at most n_seg segments cuts its work into items of
+// a wavefront: row tiles (short rows: several, so the ring's start-up is paid
+// once per ~16 records), or, where that leaves wavefronts without an item,
+// fewer row tiles or a row tile in parts whose sums the next launch adds, as
+// long as every wavefront takes one item at most.
+// One token (top-8 of 64 and the shared expert, hidden 6144, inter 2048): 576
+// row tiles of gate and up (three parts each) and 864 of down (two parts) for
+// 2048 wavefronts: 74 us a step with whole tiles, 61 us in parts.
+struct ItemCut {
+    int tiles, parts;
+};
+ItemCut item_cut(long long n_seg, int n_tensors, int tiles, int nb, int max_parts, int n_waves) {
+    ItemCut c{1, 1};
+    while (c.tiles < 4 && tiles % (2 * c.tiles) == 0 && nb * c.tiles < 16) c.tiles *= 2;
+    const long long all = n_seg * n_tensors * tiles;  // row tiles
+    while (c.tiles > 1 && all / (c.tiles / 2) <= n_waves) c.tiles /= 2;
+    while (c.tiles == 1 && c.parts < max_parts && 2 * (c.parts + 1) <= nb && all * (c.parts + 1) <= n_waves) ++c.parts;
+    return c;
+}
+// Segments a step of T tokens has at most.
+long long most_segs(int T, int E, int K, int T_sh) {
+    const long long N = (long long)T * K;
+    return std::min(N, E + N / kSegTok) + (T_sh + kSegTok - 1) / kSegTok;
+}
 
 // T_sh: shared-expert tokens (0 or T). fused: the whole step from the
 // logits (router outputs, router scratch and per-token X images in the
@@ -935,10 +991,11 @@ MoeLayout moe_layout(int T, int E, int K, int H, int I, int T_sh = 0, bool fused
     } else {
         L.act1 = off; off += L.stride1 * L.seg_max;
     }
-    L.g = off; off += align256(NS * I * 4);
-    L.u = off; off += align256(NS * I * 4);
+    const size_t rows = part_rows(NS);
+    L.g = off; off += align256(rows * I * 4);
+    L.u = off; off += align256(rows * I * 4);
     L.act2 = off; off += L.stride2 * L.seg_max;
-    L.d = off; off += align256(NS * H * 4);
+    L.d = off; off += align256(rows * H * 4);
     L.total = off;
     return L;
 }
@@ -1033,8 +1090,11 @@ hipError_t launch_moe_experts(const uint8_t* w_gate, const uint8_t* w_up, const 
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_prep_grouped<0>, dim3((N * nbH + 3) / 4), dim3(256), 0, s, X, nullptr, tok, eptr, E,
-                       nbH, 0.0f, pl, ws + L.act1, L.stride1, 0);
+                       nbH, 0.0f, pl, ws + L.act1, L.stride1, 0, 1, 0);
     const int grid = (num_cus > 0 ? num_cus : 256) * 2;
+    const int n_waves = grid * kGroupedThreads / 64, max_parts = (int)(part_rows((size_t)N) / (size_t)N);
+    const ItemCut cg = item_cut(most_segs(T, E, K, 0), 2, I / kTileRows, nbH, max_parts, n_waves);
+    const ItemCut cd = item_cut(most_segs(T, E, K, 0), 1, H / kTileRows, nbI, max_parts, n_waves);
     GroupedArgs ga{};
     ga.w[0] = w_gate;
     ga.w[1] = w_up;
@@ -1045,15 +1105,16 @@ hipError_t launch_moe_experts(const uint8_t* w_gate, const uint8_t* w_up, const 
     ga.n_tensors = 2;
     ga.nb = nbH;
     ga.tiles = I / kTileRows;
-    ga.tiles_per_item = 1;
+    ga.tiles_per_item = cg.tiles;
+    ga.parts = cg.parts;
+    ga.part_stride = (size_t)N * I;
     ga.rows = I;
     ga.pl = pl;
-    ga.ctr_index = 0;
     ga.n_exp = E;
     e = launch_timed(kProfGrouped, k_gemv_grouped, dim3(grid), dim3(kGroupedThreads), 0, s, ga);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_prep_grouped<1>, dim3((N * nbI + 3) / 4), dim3(256), 0, s, G, U, tok, eptr, E, nbI,
-                       lim, pl, ws + L.act2, L.stride2, 0);
+                       lim, pl, ws + L.act2, L.stride2, 0, cg.parts, ga.part_stride);
     GroupedArgs gd = ga;
     gd.w[0] = w_down;
     gd.w[1] = w_down;
@@ -1064,18 +1125,15 @@ hipError_t launch_moe_experts(const uint8_t* w_gate, const uint8_t* w_up, const 
     gd.n_tensors = 1;
     gd.nb = nbI;
     gd.tiles = H / kTileRows;
-    // short rows (few blocks per tile) take several tiles per item, so the
-    // ring's start-up is paid once per ~16 records
-    gd.tiles_per_item = 1;
-    while (gd.tiles_per_item < 4 && gd.tiles % (2 * gd.tiles_per_item) == 0 && gd.nb * gd.tiles_per_item < 16)
-        gd.tiles_per_item *= 2;
+    gd.tiles_per_item = cd.tiles;
+    gd.parts = cd.parts;
+    gd.part_stride = (size_t)N * H;
     gd.rows = H;
-    gd.ctr_index = 1;
     e = launch_timed(kProfGrouped, k_gemv_grouped, dim3(grid), dim3(kGroupedThreads), 0, s, gd);
     if (e != hipSuccess) return e;
     const size_t n4 = (size_t)T * H / 4;
     hipLaunchKernelGGL(k_moe_combine, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, D, wt, pl.pos, T, K, H,
-                       Y, nullptr, pl.n_seg);
+                       Y, nullptr, pl.n_seg, cd.parts, gd.part_stride);
     return hipGetLastError();
 }
 
@@ -1167,11 +1225,15 @@ hipError_t launch_moe_batch(const float* logits, int T, int E, int K, int mode, 
         if (e != hipSuccess) return e;
         const size_t n4 = (size_t)T * H / 4;
         hipLaunchKernelGGL(k_moe_combine, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, D, wt, pl.pos, T, K,
-                           H, Y, T_sh ? D + (size_t)N * H : nullptr, pl.n_seg);
+                           H, Y, T_sh ? D + (size_t)N * H : nullptr, pl.n_seg, 1, 0);
         return hipGetLastError();
     }
     // 2. gate / up of every segment (the shared expert's first)
     const int grid = (num_cus > 0 ? num_cus : 256) * 2;
+    const int n_waves = grid * kGroupedThreads / 64, max_parts = (int)(part_rows((size_t)NS) / (size_t)NS);
+    const long long segs = most_segs(T, E, K, T_sh);
+    const ItemCut cg = item_cut(segs, 2, I / kTileRows, nbH, max_parts, n_waves);
+    const ItemCut cd = item_cut(segs, 1, H / kTileRows, nbI, max_parts, n_waves);
     GroupedArgs ga{};
     ga.w[0] = w_gate;
     ga.w[1] = w_up;
@@ -1185,16 +1247,17 @@ hipError_t launch_moe_batch(const float* logits, int T, int E, int K, int mode, 
     ga.n_tensors = 2;
     ga.nb = nbH;
     ga.tiles = I / kTileRows;
-    ga.tiles_per_item = 1;
+    ga.tiles_per_item = cg.tiles;
+    ga.parts = cg.parts;
+    ga.part_stride = (size_t)NS * I;
     ga.rows = I;
     ga.pl = pl;
-    ga.ctr_index = 0;
     ga.n_exp = E;
     e = launch_timed(kProfGrouped, k_gemv_grouped, dim3(grid), dim3(kGroupedThreads), 0, s, ga);
     if (e != hipSuccess) return e;
     // 3. SwiGLU images per slot
     hipLaunchKernelGGL(k_prep_grouped<1>, dim3((NS * nbI + 3) / 4), dim3(256), 0, s, G, U, tok, eptr, E, nbI, lim,
-                       pl, ws + L.act2, L.stride2, T_sh);
+                       pl, ws + L.act2, L.stride2, T_sh, cg.parts, ga.part_stride);
     // 4. down
     GroupedArgs gd = ga;
     gd.w[0] = w_down;
@@ -1210,17 +1273,16 @@ hipError_t launch_moe_batch(const float* logits, int T, int E, int K, int mode, 
     gd.n_tensors = 1;
     gd.nb = nbI;
     gd.tiles = H / kTileRows;
-    gd.tiles_per_item = 1;
-    while (gd.tiles_per_item < 4 && gd.tiles % (2 * gd.tiles_per_item) == 0 && gd.nb * gd.tiles_per_item < 16)
-        gd.tiles_per_item *= 2;
+    gd.tiles_per_item = cd.tiles;
+    gd.parts = cd.parts;
+    gd.part_stride = (size_t)NS * H;
     gd.rows = H;
-    gd.ctr_index = 1;
     e = launch_timed(kProfGrouped, k_gemv_grouped, dim3(grid), dim3(kGroupedThreads), 0, s, gd);
     if (e != hipSuccess) return e;
     // 5. weighted combine in expert order, then the shared expert's rows
     const size_t n4 = (size_t)T * H / 4;
     hipLaunchKernelGGL(k_moe_combine, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, s, D, wt, pl.pos, T, K, H,
-                       Y, T_sh ? D + (size_t)N * H : nullptr, pl.n_seg);
+                       Y, T_sh ? D + (size_t)N * H : nullptr, pl.n_seg, cd.parts, gd.part_stride);
     return hipGetLastError();
 }
 
