@@ -145,13 +145,16 @@ def _torch():
 
 
 def _stream(stream=None):
+    if stream is not None:
+        return stream.cuda_stream
+    # the current stream's handle without a Stream object around it (2.7 us a
+    # call against 0.3, of the 6 to 8 us that the smallest kernels take)
     torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return C.c_void_p(s.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
-def _ptr(t) -> C.c_void_p:
-    return C.c_void_p(t.data_ptr())
+def _ptr(t) -> int:
+    return t.data_ptr()
 
 
 def _require_cuda(*ts):
