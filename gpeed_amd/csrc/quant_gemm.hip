@@ -17,10 +17,10 @@
 //
 // Measured, 6144 x 6144, us before (quant_rows.hip) and now:
 //   tokens     8        20       64       256      509      1024
-//   Q8_0    55 / 25  118 / 30  154 / 39  285 / 89  500 / 167  860 / 299
-//   Q3_K    53 / 31  115 / 36  152 / 45  306 / 100 515 / 203  917 / 369
-//   F16     75 / 25  131 / 28  149 / 37  285 / 75  483 / 135  848 / 235
-// No single cost bounds the large sizes: of 376 us at 1024 tokens (Q3_K), two
+//   Q8_0    55 / 25  118 / 30  154 / 40  285 / 93  500 / 165  860 / 285
+//   Q3_K    53 / 31  115 / 35  152 / 45  306 / 100 515 / 191  917 / 350
+//   F16     75 / 25  131 / 29  149 / 37  285 / 77  483 / 134  848 / 225
+// No single cost bounds the large sizes: of 376 us at 1024 tokens (Q3_K, 8 tiles), two
 // of the three MFMAs take 83, the decode 29, the X reads from LDS 43, the
 // barriers 34 (each left out alone).
 //
@@ -268,10 +268,10 @@ constexpr int kPerCu = 2;  // workgroups per CU that LDS and registers allow
 // of X a stage.
 template <int DT, int NT>
 struct SplitTile {
-    static constexpr int kSps = NT == 8 ? 1 : NT == 4 ? 2 : 4;  // steps of X a stage
+    static constexpr int kSps = NT > 4 ? 1 : NT == 4 ? 2 : 4;  // steps of X a stage
     static constexpr int kXb = NT >= 4 ? 3 : 2;                 // stages of X in LDS
     static constexpr int kStage = NT * kSps * 2 * kFrag;
-    static constexpr int kCopies = kStage / (4 * kFrag);  // copies of a stage per wavefront (NT 1, 2, 4, 8: 2, 4, 4, 4)
+    static constexpr int kCopies = (kStage / kFrag + 3) / 4;  // copies of a stage per wavefront
     static constexpr int kWBuf = Stage<DT>::kOn ? Stage<DT>::kLoads * 1024 : 16;
     // row groups in LDS per wavefront: two for few tokens, where they fit
     static constexpr int kWb = NT <= 2 && 8 * kWBuf + kXb * kStage + (int)sizeof(Tables<DT>) <= 80 * 1024 ? 2 : 1;
@@ -356,7 +356,7 @@ __global__ __launch_bounds__(256, kPerCu) void k_gemm_split(
         uint8_t* dst = xs[st % T::kXb];
 #pragma unroll
         for (int k = 0; k < T::kCopies; ++k) {
-            const int f = wave + 4 * k, u = f / (2 * SPS), v = f % (2 * SPS);  // token tile, fragment of its steps
+            const int f = min(wave + 4 * k, 2 * NT * SPS - 1), u = f / (2 * SPS), v = f % (2 * SPS);  // token tile, fragment of its steps
             const int tt = min(tm * NT + u, tt_all - 1);
             load_lds16(xf + (((size_t)tt * n_chunk + c) * 8 + 2 * s0 + v) * kFrag + lane * 16, dst + f * kFrag);
         }
@@ -550,9 +550,14 @@ int pass_tokens(int in_dim, int n_tok) {
 }
 
 // The launch of one product: 16 nt tokens per workgroup and splits of K.
-// nt is the largest tile the tokens fill by more than half for which the
-// tiles and splits make 256 workgroups (one per CU), the splits what fills
-// the kPerCu slots of 256 CUs, each of at least two chunks.
+// Up to 64 tokens the least of 1, 2, 4 tiles that holds them, fewer where the
+// tiles and splits would not make a workgroup for each of 256 CUs. Above, of
+// 4, 6, 7 and 8 tiles the one with the least time: rounds of the kPerCu slots
+// of 256 CUs times chunks of a split times about 1.5 + 0.78 nt us (measured,
+// Q3_K: 4.6 at 4 tiles, 7.7 at 8), and the splits' sums written and read.
+// 6144 rows (Q3_K, us with 8 tiles and with the choice): 96 tokens 6 tiles 60
+// and 54, 200 tokens 7 tiles 98 and 92, 509 tokens 7 tiles 204 and 193, 1024
+// tokens 7 tiles 372 and 351.
 constexpr int kMaxSplit = 16;
 struct RowsPlan {
     int nt, splits;
@@ -560,11 +565,25 @@ struct RowsPlan {
 RowsPlan rows_plan(int in_dim, int out_dim, int n_tok) {
     const int n_chunk = (in_dim + kChunk - 1) / kChunk;
     const long long tn = ((long long)out_dim + 127) / 128, most = std::max(1, std::min(kMaxSplit, n_chunk / 2));
-    for (int nt = n_tok <= 16 ? 1 : n_tok <= 32 ? 2 : n_tok <= 64 ? 4 : 8;; nt /= 2) {
-        const long long wg = tn * ((n_tok + 16 * nt - 1) / (16 * nt));
-        if (nt == 1 || wg * most >= 256)
-            return {nt, (int)std::max<long long>(1, std::min<long long>(most, 256ll * kPerCu / wg))};
+    const auto groups = [&](int nt) { return tn * ((n_tok + 16 * nt - 1) / (16 * nt)); };
+    const auto splits = [&](int nt) {
+        return (int)std::max<long long>(1, std::min<long long>(most, 256ll * kPerCu / groups(nt)));
+    };
+    if (n_tok <= 64 || groups(4) * most < 256) {
+        int nt = n_tok <= 16 ? 1 : n_tok <= 32 ? 2 : 4;
+        while (nt > 1 && groups(nt) * most < 256) nt /= 2;
+        return {nt, splits(nt)};
     }
+    RowsPlan best{8, 1};
+    double least = 0.0;
+    for (int nt : {8, 7, 6, 4}) {
+        const int s = splits(nt);
+        const double rounds = (double)((groups(nt) * s + 256 * kPerCu - 1) / (256 * kPerCu));
+        const double us = rounds * ((n_chunk + s - 1) / s) * (1.5 + 0.78 * nt) +
+                          (s > 1 ? 3.0 + 8e-6 * s * (double)n_tok * out_dim / 4.0 : 0.0);
+        if (least == 0.0 || us < 0.97 * least) best = {nt, s}, least = us;
+    }
+    return best;
 }
 
 struct RowsWs {  // the workspace of one pass
@@ -621,6 +640,8 @@ hipError_t rows_gemm_dt(const uint8_t* w, size_t rb, int in_dim, int out_dim, co
             case 1: e = gemm_split_nt<DT, 1>(w, rb, in_dim, out_dim, r, Xt, n, Yt, pl.splits, s); break;
             case 2: e = gemm_split_nt<DT, 2>(w, rb, in_dim, out_dim, r, Xt, n, Yt, pl.splits, s); break;
             case 4: e = gemm_split_nt<DT, 4>(w, rb, in_dim, out_dim, r, Xt, n, Yt, pl.splits, s); break;
+            case 6: e = gemm_split_nt<DT, 6>(w, rb, in_dim, out_dim, r, Xt, n, Yt, pl.splits, s); break;
+            case 7: e = gemm_split_nt<DT, 7>(w, rb, in_dim, out_dim, r, Xt, n, Yt, pl.splits, s); break;
             default: e = gemm_split_nt<DT, 8>(w, rb, in_dim, out_dim, r, Xt, n, Yt, pl.splits, s); break;
         }
         if (e != hipSuccess) return e;

@@ -69,6 +69,18 @@ def test_partial_last_chunk(gpu, dt, in_dim):
     assert rel_err(Y, oracle.matmul_rows(dt, w, 0, in_dim, rows, X)) < TIGHT
 
 
+@pytest.mark.parametrize("dt", [1, 11])
+@pytest.mark.parametrize("n_tok", [66, 96, 128, 200, 300])
+def test_token_tiles_vs_float32(gpu, dt, n_tok):
+    """A 6144 x 6144 product at the token counts where the launch takes 4, 6, 7
+    and 8 token tiles of 16 a workgroup, partly filled ones among them."""
+    n = 6144
+    w = dev(synth.quant_matrix(68, dt, dt, n, n).reshape(-1), gpu)
+    X = dev(synth.normal(68, n_tok, n_tok * n).reshape(n_tok, n), gpu)
+    Y = G.matmul_rows(dt, w, n, 0, n, n, X).cpu().numpy()
+    assert rel_err(Y, rows_f32(dt, w, n, 0, n, n, X).cpu().numpy()) < 2 * TIGHT  # (both sides' order)
+
+
 @pytest.mark.parametrize("dt", TYPES)
 @pytest.mark.parametrize("n_tok", [8, 40, 300])
 def test_no_less_precise_than_float32(gpu, dt, n_tok):
