@@ -26,27 +26,6 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// The replicated grid table, built by a workgroup of kThreads threads: the
-// codebook words are fetched first (grid_words), the LDS writes done later
-// (grid_table_store) so that loads issued in between stay in flight.
-template <int kThreads>
-struct GridWords {
-    static constexpr int kPer = (1024 + kThreads - 1) / kThreads;
-    uint32_t v[kPer];
-};
-
-template <int kThreads>
-__device__ __forceinline__ void grid_words(GridWords<kThreads>& gw, int tid) {
-#pragma unroll
-    for (int i = 0; i < GridWords<kThreads>::kPer; ++i)
-        gw.v[i] = kIq3xxsGrid[((tid + i * kThreads) >> 2) & 255];
-}
-
-__device__ __forceinline__ uint32_t f16_pair_of_bytes(uint32_t lo, uint32_t hi) {
-    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)lo) |
-           ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)hi) << 16);
-}
-
 // Exact fp16 bit pattern of a small non-negative integer (< 2048).
 constexpr uint32_t f16_bits_of_uint(uint32_t a) {
     if (a == 0) return 0;
@@ -62,8 +41,9 @@ constexpr uint32_t grid_f16_pair(int idx, int half) {
            (f16_bits_of_uint((kIq3xxsGrid[idx] >> (16 * half + 8)) & 255u) << 16);
 }
 
-// The replicated grid table written from immediate operands (no memory
-// loads, so no wait behind other loads): wavefront w of W writes entries
+// The replicated grid table (entry idx, replica r at byte (idx << 8) | (r <<
+// 3): 4 unsigned fp16), written from immediate operands (no memory loads, so
+// no wait behind other loads): wavefront w of W writes entries
 // [w*256/W, (w+1)*256/W), two per store (lanes 0-31 the even entry's 32
 // replicas, lanes 32-63 the odd one's).
 template <int W>
@@ -83,24 +63,6 @@ __device__ __forceinline__ void grid_table_literal(uint8_t* tbl, int wave, uint3
             });
         }
     });
-}
-
-// Entry idx, replica r at byte (idx << 8) | (r << 3): 4 unsigned fp16.
-template <int kThreads>
-__device__ __forceinline__ void grid_table_store(uint8_t* tbl, const GridWords<kThreads>& gw, int tid) {
-#pragma unroll
-    for (int i = 0; i < GridWords<kThreads>::kPer; ++i) {
-        const int it = tid + i * kThreads;
-        if (it < 1024) {
-            const int idx = it >> 2, q4 = it & 3;
-            const uint32_t v = gw.v[i];
-            const uint32_t h01 = f16_pair_of_bytes(v & 255u, (v >> 8) & 255u);
-            const uint32_t h23 = f16_pair_of_bytes((v >> 16) & 255u, v >> 24);
-            u32x4_t* dst = reinterpret_cast<u32x4_t*>(tbl + (idx << 8) + q4 * 64);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) dst[j] = u32x4_t{h01, h23, h01, h23};
-        }
-    }
 }
 
 // One record as a lane holds it: its row's 24 dwords and d, the NP
